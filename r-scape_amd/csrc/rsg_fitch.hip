@@ -474,14 +474,6 @@ __global__ void __launch_bounds__(NT) k_fitch_down_replay(const int4 *__restrict
   else                        down_block<NT>(dent[blockIdx.x - nrep], N, L, ax, seeds, flag, mask, all, rs, nsub);
 }
 
-// Orders a wave's global stores before its later loads (lanes exchange data through memory;
-// the waves of a block work on different branches and never wait for each other).
-__device__ __forceinline__ void wave_sync()
-{
-  __threadfence_block();
-  __builtin_amdgcn_wave_barrier();
-}
-
 // The replay for rows too long for LDS (L > FITCH_LDS_L): one wave per branch.  For each
 // old symbol: the parent's positions holding it (ascending, ballot compaction) in cols_all (L ints
 // per wave slot, 2 maxw slots per replicate), the swaps, whose indices the 64 lanes draw ahead,

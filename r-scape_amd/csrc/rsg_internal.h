@@ -86,6 +86,14 @@ __device__ __forceinline__ unsigned onehot4(unsigned codes)
   return __builtin_amdgcn_perm(0u, 0x08040201u, (codes & 0x03030303u) | (big >> 5));
 }
 
+// Orders what the lanes of a wave exchange through memory (LDS or global): stores before it are seen by
+// every lane's loads after it.  For waves that share data with no other wave of their work group.
+__device__ __forceinline__ void wave_sync()
+{
+  __threadfence_block();
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Packs the 128-sequence x 128-column block at (s0, c0) with 256 threads: the codes come in as
 // dwords of four columns (unaligned: L is any number; 16 loads in flight per thread), cross an
 // LDS tile, and leave as 16-byte stores, two columns per thread: consecutive threads take

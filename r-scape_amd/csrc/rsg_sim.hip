@@ -233,6 +233,7 @@ k_evolve_level(const SimItem *__restrict__ items, const int4 *__restrict__ ent, 
   const int64_t L = it.L, v = e.y;
   if (64 * (int64_t)blockIdx.y >= L) return;
   if (lane < 24) th[wave][lane / 12][lane % 12 / 3][lane % 3] = cdf[(it.tree_off + v) * 24 + lane];
+  wave_sync();                                 // every lane reads what these 24 wrote
   const int dl = e.z, dr = e.w;
   const uint8_t *par = seqs + it.seq_off + v * L;
   uint8_t *out0 = (dl > 0) ? seqs + it.seq_off + (int64_t)dl * L : leaves + it.leaf_off + (int64_t)(-dl) * L;

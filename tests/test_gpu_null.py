@@ -42,6 +42,23 @@ def test_simulation_matches_oracle(ctx, N, L, gap):
     assert got.max() <= 4
 
 
+@pytest.mark.parametrize("L", [1, 23, 24, 25, 64, 65, 257])
+@pytest.mark.parametrize("N", [2, 6, 7, 41])
+def test_simulation_branch_tables(ctx, N, L):
+    """Each wave of the evolution keeps its own node's thresholds: trees whose levels hold 1 to 20
+    nodes of branches from 0.001 to 3 (thresholds of the four waves of a work group far apart; the
+    last work group of a level part empty), and rows shorter than the lanes that load the thresholds.
+    The tolerance of the tests above (a threshold may differ from the host's by a few units of 2^-32)."""
+    m = NL.gtr_model(PI)
+    rng = np.random.default_rng(100 * N + L)
+    tree = NL.yule_tree(N, 0.2, seed=N + L)
+    for k in ("ld", "rd"):
+        tree[k] = 10.0 ** rng.uniform(-3, np.log10(3.0), N - 1)
+    j = NL.Job(tree, L, m, seed=77 + L, stream=3, gapfrac=0.1)
+    got = NL.simulate(ctx, j)
+    assert np.mean(got != oracle.evolve_gtr(j.tree, j.L, m, j.seed, j.stream, int(0.1 * 2 ** 32))) < 1e-5
+
+
 def test_simulation_distribution(ctx):
     """Leaf composition is stationary; mean pairwise difference follows the tree."""
     m = NL.gtr_model(PI)
