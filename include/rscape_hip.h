@@ -82,9 +82,9 @@ int         rsg_ctx_set_gram_split(rsg_ctx *ctx, int on);
  * by per-XCD tile queues (longest K first); 0 launches one work group per tile.  Results are
  * identical (no reference counterpart). */
 int         rsg_ctx_set_batch_persistent(rsg_ctx *ctx, int on);
-/* How long rsg_cov_Calculate_noalloc spins on its completion stamp in pinned host memory before
- * it waits in a stream synchronisation instead (default 2000 microseconds; 0 = always
- * synchronise, as rsg_cov_Calculate does).  Results are the same either way (no reference counterpart). */
+/* How long rsg_cov_Calculate and rsg_cov_Calculate_noalloc spin on their completion stamp in pinned
+ * host memory before they synchronise the stream, which they do in any case (default 0 microseconds: no
+ * spin).  Results are the same either way (no reference counterpart). */
 int         rsg_ctx_set_stamp_wait(rsg_ctx *ctx, int microseconds);
 /* Counter calibration (no reference counterpart): runs the plain copy kernel
  * k_copy_probe over `bytes` (multiple of 16) three times, reading and writing `bytes` per

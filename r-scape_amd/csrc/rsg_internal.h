@@ -272,9 +272,9 @@ struct rsg_ctx {
   double      *d_hres = nullptr;        // h_pinned as the device addresses it
   int          res_on_host = 0;
   // completion stamp: the min / max reduction writes hstamp to h_pinned[63] after the result
-  // block (system-scope release), so the caller can wait for it without a stream synchronisation
+  // block (system-scope release)
   unsigned long long hstamp = 0;
-  int          stamp_wait_us = 2000;    // spin on the stamp this long, then synchronise the stream
+  int          stamp_wait_us = 0;       // spin on the stamp this long before the stream is synchronised
   void        *d_small = nullptr;       // 64 KB of device scratch for small per-call tables
   // set for the duration of an allocation-free call (rsg_noalloc.hip): the Gram takes this
   // 32 x 32-column tile list instead of its cached one, and d_red is not grown past red_cap

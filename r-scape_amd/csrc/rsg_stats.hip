@@ -335,7 +335,7 @@ static int launch_stat_f32_fixed(rsg_ctx *c, const StatArgs &A, int kind, int cl
 // (min, max) of n block partials into out[0..1]; one block of 256 threads, four partials per
 // thread loaded at once, then block_minmax256.  With hout != nullptr out[0..4] (min, max and the
 // flags and COVavg the chain left in out[2..4]) also go to hout, host memory, followed (after a
-// system-scope release) by the completion stamp in hout[63], which the caller waits for.
+// system-scope release) by the completion stamp in hout[63].
 __global__ void __launch_bounds__(256) k_reduce_minmax(const double *__restrict__ part, int n, double *__restrict__ out,
                                                        double *__restrict__ hout, unsigned long long stamp)
 {

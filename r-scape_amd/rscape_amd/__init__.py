@@ -254,8 +254,8 @@ class Context:
         self.L.rsg_ctx_set_batch_persistent(self.h, 1 if on else 0)
 
     def set_stamp_wait(self, microseconds):
-        """How long an allocation-free scoring call spins on its completion stamp before it
-        synchronises the stream instead (0: always synchronise, as the others do)."""
+        """How long a scoring call spins on its completion stamp before it synchronises the
+        stream (0, the default: not at all)."""
         self.L.rsg_ctx_set_stamp_wait(self.h, int(microseconds))
 
     def graph_reuses(self):
