@@ -260,7 +260,8 @@ struct rsg_ctx {
   int          bexec_hits = 0;          // replays that reused the cached graph (for tests)
   void        *d_hits = nullptr;  size_t hits_cap = 0;   // hit-list compaction (grow-only, entries)
   void        *h_hits = nullptr;                          // its pinned host mirror, same capacity
-  void        *d_rank = nullptr, *h_rank = nullptr;       // rank histogram: slices and list, pinned results
+  void        *d_rank = nullptr, *h_rank = nullptr;       // rank histogram: slices, list, counters, pinned results
+  int          rank_dirty = 0;                            // its dense counters to clear before the next call
   // small reusable device scratch (reductions)
   double      *d_red = nullptr;  size_t red_cap = 0;
   int         *d_flag = nullptr;

@@ -87,26 +87,35 @@ extern "C" double rsg_width(double maxCOV, double minCOV, double bmin, double w_
 // ---------------------------------------------------------------- device histogram
 // Scores crowd into the bins just above the smallest one (the background: a few hundred bins),
 // while the largest score sets how many bins there are (145 000 for GT at N = 5000, L = 1500).  A
-// work group counts the RANK_WIN bins from b0 (the smallest score's bin) in LDS and leaves them as
-// its slice of `part`; the scores past them are few (the covarying pairs) and go to a list of
-// bin indices, or, when the list is too short, to the dense counters (`dense`).  Counting every
-// score of such a histogram in global atomics instead serialises on the background's bins:
-// 4720 us at N = 5000 x L = 1500 and 55.6 ms at L = 5000, against 14 and 33 us here (with
-// k_hist_sum).  Bound by the latency of one pass over the upper triangle and its FP64 divisions.
+// work group counts the `win` bins from b0 (the smallest score's bin) in LDS and leaves them as
+// its slice of `part`: all bins where they are RANK_WIN at most, else RANK_NEAR of them.  The scores past
+// them are few where a correction has taken the background off and bins are wide (the covarying
+// pairs): the work group lists their bins, `slice` of them (its part of `list`; gcount: how many there
+// were).  What does not fit (a background wider than the window) goes to the counters of all bins,
+// `dense`, in the same pass, and k_hist_sum then leaves everything there.
+// Counting every score in global atomics instead serialises on the background's bins: GT with APC 4690 us
+// at 5000 x 1500 and 19.9 ms at 12000 x 3000, 15 and 20 us here (with k_hist_sum); without a correction
+// 220 and 850 us, 15 and 20 here; the same in bins a tenth as wide, where a fifth of the scores are past the
+// window, 54 and 200 us, 31 and 94 here.
+// Bound by the latency of one pass over the upper triangle and its FP64 divisions.
 // Work group g takes the row pairs p = g, g + G, ... (rows p and L - 1 - p, L - 1 elements
 // together, so all pairs cost the same).
-#define RANK_WIN  8192        // bins counted in LDS (32 KiB)
-#define RANK_LIST 65536       // list of the bins past the window
-#define RANK_GRID 256         // work groups at most: one per CU, each leaves RANK_WIN counters
+#define RANK_WIN  16384       // bins counted in LDS at most (64 KiB)
+#define RANK_NEAR 8192        // and where they are not all: half the slices to write and add (2 us at 203 columns)
+#define RANK_LIST 131072      // list of the bins past the window, over all work groups
+#define RANK_GRID 256         // work groups at most: one per CU, each leaves `win` counters
+#define RANK_DENSE (1 << 18)  // bins of the context's dense counters (2 MiB, zero between calls)
 __global__ void __launch_bounds__(1024)
-k_hist(const double *__restrict__ cov, int64_t L, double bmin, double w, int nb, int b0, int win,
-       unsigned *__restrict__ part, unsigned *__restrict__ nover, int *__restrict__ list,
-       unsigned long long *__restrict__ dense)
+k_hist(const double *__restrict__ cov, int64_t L, double bmin, double w, int nb, int b0, int win, int slice,
+       unsigned *__restrict__ part, int *__restrict__ gcount, int *__restrict__ list, unsigned long long *__restrict__ dense)
 {
-  __shared__ unsigned lh[RANK_WIN];
+  extern __shared__ unsigned lh[];
+  __shared__ int nlist;
   for (int b = threadIdx.x; b < win; b += 1024) lh[b] = 0u;
+  if (threadIdx.x == 0) nlist = 0;
   __syncthreads();
   const double floor_v = bmin + w;
+  int *mine = list + (int64_t)blockIdx.x * slice;
   for (int64_t p = blockIdx.x; 2 * p < L; p += gridDim.x) {
     const int64_t n0 = L - 1 - p, tot = (2 * p == L - 1) ? n0 : L - 1;
     const double *r0 = cov + p * L + p + 1, *r1 = cov + (L - 1 - p) * L + 1;
@@ -125,66 +134,90 @@ k_hist(const double *__restrict__ cov, int64_t L, double bmin, double w, int nb,
         b = (b < 0) ? 0 : ((b >= nb) ? nb - 1 : b);               // cannot happen: bmax = maxCOV + 5w
         const unsigned k = (unsigned)(b - b0);
         if (k < (unsigned)win) atomicAdd(&lh[k], 1u);
-        else if (dense) atomicAdd(&dense[b], 1ull);
         else {
-          const unsigned o = atomicAdd(nover, 1u);
-          if (o < RANK_LIST) list[o] = b;
+          const int o = atomicAdd(&nlist, 1);
+          if (o < slice) mine[o] = b;
+          else atomicAdd(&dense[b], 1ull);
         }
       }
     }
   }
   __syncthreads();
-  for (int b = threadIdx.x; b < win; b += 1024) part[(int64_t)blockIdx.x * RANK_WIN + b] = lh[b];
+  for (int b = threadIdx.x; b < win; b += 1024) part[(int64_t)blockIdx.x * win + b] = lh[b];
+  if (threadIdx.x == 0) gcount[blockIdx.x] = nlist;
 }
 
-// The window's counts summed over the work groups' slices, into pinned host memory with the list
-// and its length: block k takes bins 64 k .. 64 k + 63, wave q of 16 the slices q, q + 16, ...
-// (all its loads in flight at once; with four waves per block, 64 loads in turn, it took 17.5 us).
-// The last read of nover is here, so it is cleared for the next call.
+// The window's counts summed over the work groups' slices: block k takes bins 64 k .. 64 k + 63, wave q
+// of 16 the slices q, q + 16, ... (all its loads in flight at once; with four waves per block, 64 loads in
+// turn, it took 17.5 us).  When every list held its work group's bins, the sums go to pinned host memory
+// and the last block appends the lists there one after another; else sums and lists go to `dense`.
+// *hlen: the listed bins, or -1.
 __global__ void __launch_bounds__(1024)
-k_hist_sum(const unsigned *__restrict__ part, int ng, int win, unsigned *__restrict__ nover, const int *__restrict__ list,
-           unsigned long long *__restrict__ hwin, int *__restrict__ hlist, unsigned *__restrict__ hnover)
+k_hist_sum(const unsigned *__restrict__ part, int ng, int b0, int win, int slice, const int *__restrict__ gcount,
+           const int *__restrict__ list, unsigned long long *__restrict__ dense, unsigned long long *__restrict__ hwin,
+           int *__restrict__ hlist, int *__restrict__ hlen)
 {
   __shared__ unsigned long long sh[16][64];
-  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, b = blockIdx.x * 64 + lane;
+  __shared__ int off[RANK_GRID + 1], wtot[RANK_GRID / 64];
+  const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6, b = blockIdx.x * 64 + lane;
   unsigned v[RANK_GRID / 16];
 #pragma unroll
   for (int k = 0; k < RANK_GRID / 16; k++) {
     const int g = q + 16 * k;
-    v[k] = (b < win && g < ng) ? part[(int64_t)g * RANK_WIN + b] : 0u;
+    v[k] = (b < win && g < ng) ? part[(int64_t)g * win + b] : 0u;
   }
+  const int n = tid < ng ? gcount[tid] : 0;
+  int x = n;                                               // list lengths, inclusive over the wave
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) { const int y = __shfl_up(x, d, 64); if (lane >= d) x += y; }
+  if (q < RANK_GRID / 64 && lane == 63) wtot[q] = x;
   unsigned long long s = 0ull;
 #pragma unroll
   for (int k = 0; k < RANK_GRID / 16; k++) s += v[k];
   sh[q][lane] = s;
-  __syncthreads();
+  const int spill = __syncthreads_or(n > slice);
   if (q == 0 && b < win) {
 #pragma unroll
     for (int k = 1; k < 16; k++) s += sh[k][lane];
-    hwin[b] = s;
+    (spill ? dense + b0 : hwin)[b] = s;
   }
-  if (blockIdx.x == gridDim.x - 1) {
-    const unsigned n = *nover, m = n < RANK_LIST ? n : RANK_LIST;
-    for (unsigned k = threadIdx.x; k < m; k += 1024) hlist[k] = list[k];
-    __syncthreads();
-    if (threadIdx.x == 0) { *hnover = n; *nover = 0u; }
+  if (spill) {
+    for (int64_t e = (int64_t)blockIdx.x * 1024 + tid; e < (int64_t)ng * slice; e += (int64_t)gridDim.x * 1024) {
+      const int64_t g = e / slice;
+      if (e - g * slice < gcount[g]) atomicAdd(&dense[list[e]], 1ull);
+    }
+    if (blockIdx.x == 0 && tid == 0) *hlen = -1;
+    return;
   }
+  if (blockIdx.x != gridDim.x - 1) return;
+  if (tid < RANK_GRID) {
+    for (int k = 0; k < q; k++) x += wtot[k];
+    off[tid + 1] = x;
+  }
+  if (tid == 0) off[0] = 0;
+  __syncthreads();
+  const int len = off[RANK_GRID];
+  for (int e = tid; e < len; e += 1024) {
+    int g = 0;                                             // the last list that starts at or before e
+#pragma unroll
+    for (int d = RANK_GRID / 2; d > 0; d >>= 1) if (off[g + d] <= e) g += d;
+    hlist[e] = list[(int64_t)g * slice + e - off[g]];
+  }
+  if (tid == 0) *hlen = len;
 }
 
-// The context's buffers for it, made at the first call: on the device the slices, the list and its
-// length (8.3 MB), pinned on the host the window, the list and its length (0.3 MB).
+// The context's buffers for it, made at the first call: on the device the slices, the lists, their
+// lengths and the dense counters (20 MB), pinned on the host the window, the list and its length (0.7 MB).
+static constexpr size_t RANK_SLICES = sizeof(unsigned) * (size_t)RANK_GRID * RANK_WIN, RANK_LISTB = sizeof(int) * RANK_LIST,
+                        RANK_COUNTS = sizeof(int) * RANK_GRID, RANK_DENSEB = sizeof(unsigned long long) * RANK_DENSE;
 static int ensure_rank(rsg_ctx *c, char *errbuf)
 {
   if (c->h_rank) return RSG_OK;
   if (!c->d_rank) {
-    HIPCHK(hipMalloc(&c->d_rank, sizeof(unsigned) * (size_t)RANK_GRID * RANK_WIN + sizeof(int) * RANK_LIST + 64));
-    unsigned *nover = (unsigned *)c->d_rank + (size_t)RANK_GRID * RANK_WIN + RANK_LIST;
-    if (hipMemsetAsync(nover, 0, 64, c->stream) != hipSuccess) {
-      hipFree(c->d_rank); c->d_rank = nullptr;
-      return rsg_fail(errbuf, "rsg_cov_RankHist: memset failed");
-    }
+    HIPCHK(hipMalloc(&c->d_rank, RANK_SLICES + RANK_LISTB + RANK_COUNTS + RANK_DENSEB));
+    c->rank_dirty = RANK_DENSE;
   }
-  HIPCHK(hipHostMalloc(&c->h_rank, sizeof(unsigned long long) * RANK_WIN + sizeof(int) * RANK_LIST + 64, hipHostMallocDefault));
+  HIPCHK(hipHostMalloc(&c->h_rank, sizeof(unsigned long long) * RANK_WIN + RANK_LISTB + 64, hipHostMallocDefault));
   return RSG_OK;
 }
 
@@ -217,37 +250,42 @@ extern "C" int rsg_cov_RankHist(rsg_ctx *c, rsg_msa *m, double bmin, double w, d
   h->n = h->Nc = h->No = npairs;
   if (npairs == 0) { h->imin = h->nb; h->imax = -1; h->cmin = h->nb; h->xmin = DBL_MAX; h->xmax = -DBL_MAX; }
 
-  const int b0 = std::min(std::max(bmin_b, 0), nb - 1), win = std::min(nb - b0, RANK_WIN);
-  const int grid = (int)std::min<int64_t>(RANK_GRID, (L + 1) / 2);
-  unsigned *part = (unsigned *)c->d_rank, *nover = part + (size_t)RANK_GRID * RANK_WIN + RANK_LIST;
-  int *list = (int *)(part + (size_t)RANK_GRID * RANK_WIN);
-  unsigned long long *hwin = (unsigned long long *)c->h_rank, *d_obs = nullptr;
+  const int b0 = std::min(std::max(bmin_b, 0), nb - 1), win = (nb - b0 <= RANK_WIN) ? nb - b0 : RANK_NEAR;
+  const int grid = (int)std::min<int64_t>(RANK_GRID, (L + 1) / 2), slice = RANK_LIST / grid;
+  unsigned *part = (unsigned *)c->d_rank;
+  int *list = (int *)((char *)part + RANK_SLICES), *gcount = (int *)((char *)list + RANK_LISTB);
+  unsigned long long *hwin = (unsigned long long *)c->h_rank;
   int *hlist = (int *)(hwin + RANK_WIN);
-  unsigned *hnover = (unsigned *)(hlist + RANK_LIST);
-  auto count = [&](unsigned long long *dense) -> hipError_t {
+  volatile int *hlen = hlist + RANK_LIST;
+  // counters of all bins for what the lists do not hold: the context's, cleared again before the next
+  // call once they have been used, or a block of their own for more bins
+  RsgTmp tmp(c);
+  unsigned long long *dense = (unsigned long long *)((char *)gcount + RANK_COUNTS);
+  int clear = c->rank_dirty;
+  hipError_t e = hipSuccess;
+  if (nb > RANK_DENSE) { clear = nb; e = tmp.get(&dense, sizeof(unsigned long long) * (size_t)nb); }
+  if (e == hipSuccess && clear) e = hipMemsetAsync(dense, 0, sizeof(unsigned long long) * (size_t)clear, c->stream);
+  if (e == hipSuccess) {
+    if (nb <= RANK_DENSE) c->rank_dirty = nb;
     int t;
     rsg_tstart(c, "hist", &t);
-    hipLaunchKernelGGL(k_hist, dim3((unsigned)grid), dim3(1024), 0, c->stream, m->d_cov, L, bmin, w, nb, b0, win, part, nover,
-                       list, dense);
-    hipLaunchKernelGGL(k_hist_sum, dim3((unsigned)((win + 63) / 64)), dim3(1024), 0, c->stream, part, grid, win, nover, list,
-                       hwin, hlist, hnover);
+    hipLaunchKernelGGL(k_hist, dim3((unsigned)grid), dim3(1024), sizeof(unsigned) * (size_t)win, c->stream, m->d_cov, L, bmin, w,
+                       nb, b0, win, slice, part, gcount, list, dense);
+    hipLaunchKernelGGL(k_hist_sum, dim3((unsigned)((win + 63) / 64)), dim3(1024), 0, c->stream, part, grid, b0, win, slice, gcount,
+                       list, dense, hwin, hlist, (int *)hlen);
     rsg_tstop(c, t);
-    return hipGetLastError();
-  };
-  hipError_t e = count(nullptr);
+    e = hipGetLastError();
+  }
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  if (e == hipSuccess && *hnover > RANK_LIST) {           // too many scores past the window: again, into all bins
-    e = hipMalloc(&d_obs, sizeof(unsigned long long) * (size_t)nb);
-    if (e == hipSuccess) e = hipMemsetAsync(d_obs, 0, sizeof(unsigned long long) * (size_t)nb, c->stream);
-    if (e == hipSuccess) e = count(d_obs);
-    if (e == hipSuccess) e = hipMemcpyAsync(h->obs, d_obs, sizeof(uint64_t) * (size_t)nb, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess && *hlen < 0) {
+    e = hipMemcpyAsync(h->obs, dense, sizeof(uint64_t) * (size_t)nb, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (d_obs) hipFree(d_obs);
   } else if (e == hipSuccess) {
-    for (unsigned k = 0; k < *hnover; k++) h->obs[hlist[k]]++;
+    if (nb <= RANK_DENSE) c->rank_dirty = 0;
+    for (int b = 0; b < win; b++) h->obs[b0 + b] = hwin[b];
+    for (int k = 0; k < *hlen; k++) h->obs[hlist[k]]++;
   }
   if (e != hipSuccess) { rsg_hist_destroy(h); return rsg_fail(errbuf, "rsg_cov_RankHist: %s", hipGetErrorString(e)); }
-  for (int b = 0; b < win; b++) h->obs[b0 + b] += hwin[b];
   *ret = h;
   return RSG_OK;
 }

@@ -46,6 +46,26 @@ def test_rank_histogram_wide(ctx, N, L, w):
         same_hist(m.rank_hist(-10.0, w), oracle.rank_hist(cov, L, mx, -10.0, w))
 
 
+@pytest.mark.parametrize("N,L,bins", [(60, 70, 16378), (60, 70, 16380), (60, 70, 16384), (60, 70, 16390),   # all in LDS, or the near half
+                                      (50, 420, 40000), (50, 600, 240000),      # lists that hold them, lists that do not
+                                      (50, 600, 2000000)])                      # and more bins than the context's counters
+def test_rank_histogram_spread(ctx, N, L, bins):
+    """Scores spread over many times the bins counted in LDS, as GT's are without a correction: the
+    matrix is read once whatever becomes of the scores past them (one timed pass per call; a pass that is
+    thrown away and repeated made these slower than counting them all in memory), and the bins equal the
+    oracle's, also after calls that used the counters of all bins, with more and with fewer bins."""
+    m, cov, mn, mx = scored(ctx, synth.random_msa(N, L, np.random.default_rng(L), gap=0.1), "GT")
+    w = (mx - mn) / (bins - 6)
+    ref = {x: oracle.rank_hist(cov, L, mx, -10.0, x) for x in (w, 3 * w, 0.05)}
+    for x in (w, 3 * w, w, 0.05, w):
+        ctx.set_timing(True)
+        g = m.rank_hist(-10.0, x)
+        passes = [t for t in ctx.timings() if t[0] == "hist"]
+        ctx.set_timing(False)
+        same_hist(g, ref[x])
+        assert len(passes) == 1
+
+
 def null_replicates(ctx, n=4, seed=0):
     """Score unstructured replicate alignments; return (gpu histograms, oracle histograms)."""
     rng = np.random.default_rng(seed)
