@@ -11,9 +11,9 @@
 #include <thread>
 #include <memory>
 #include <mutex>
-#include <unordered_map>
 #include <algorithm>
 #include "../../include/rscape_hip.h"
+#include "rsg_pool.h"
 
 #define RSG_MAX_TIMERS 64
 
@@ -206,36 +206,6 @@ __device__ __forceinline__ void pack_block(const uint8_t *__restrict__ ax, int64
 }
 #endif
 
-// Device blocks of short-lived objects, kept for the next ones: hipMalloc and hipFree of a dozen
-// buffers cost more than scoring a family does (score of 600 x 300 on a new alignment object,
-// R-scape's own call: 236 us with them, 174 us without).  A block put back is handed out again for
-// a request of its size class; at most RSG_POOL_KEEP bytes are kept (the rest, and blocks over
-// RSG_POOL_BLOCK, go back to the device at once), all of them are given back with the context, and
-// by every pool when an allocation of the library fails.  Any thread may call.
-// A pool does not wait for the device: its user keeps one of two rules.  `tmp` of a context holds
-// blocks that only work on that context's stream touches (RsgTmp), so stream order covers their
-// reuse; `pool` holds blocks of alignments, which any context may have used: they are put back
-// when the device is idle (as hipFree waits for it).
-#define RSG_POOL_KEEP  ((size_t)1 << 30)
-#define RSG_POOL_BLOCK ((size_t)1 << 28)
-#define RSG_POOL_COUNT 256               // idle blocks at most
-struct RsgPool {
-  RsgPool();
-  ~RsgPool();
-  hipError_t get(void **p, size_t bytes);
-  void put(void *p);
-  void close();                          // gives back the idle blocks and keeps none from here on
-  void trim();                           // gives back the idle blocks
-private:
-  std::mutex mu;
-  std::unordered_map<void *, size_t> used;            // size classes of the blocks handed out
-  std::vector<std::pair<size_t, void *>> idle;
-  size_t kept = 0;
-  bool open = true;
-};
-// hipMalloc; when it fails, again after every pool has given back its idle blocks
-hipError_t rsg_dev_malloc(void **p, size_t bytes);
-
 struct rsg_timer { const char *name; hipEvent_t a, b; double host_ms; };   // host_ms >= 0: a host phase
 
 struct rsg_ctx {
@@ -297,6 +267,7 @@ struct RsgTmp {
   template <typename T> hipError_t get(T **out, size_t bytes)
   {
     void *q = nullptr;
+    try { p.reserve(p.size() + 1); } catch (const std::bad_alloc &) { return hipErrorOutOfMemory; }
     const hipError_t e = c->tmp.get(&q, bytes);
     if (e == hipSuccess) { p.push_back(q); *out = (T *)q; }
     return e;
