@@ -553,7 +553,7 @@ struct Buf {
   template <typename T> bool get(T **o, size_t n)
   {
     void *q = nullptr;
-    if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) return false;
+    if (rsg_dev_malloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) return false;
     p.push_back(q); *o = (T *)q;
     return true;
   }

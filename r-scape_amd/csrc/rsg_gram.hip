@@ -929,7 +929,7 @@ static const int2 *tile_list(int device, int64_t L, int BI, int BJ, int *ntiles,
       if (bi * BI < jmax) v.push_back(make_int2((int)bi, (int)bj));
     }
   int2 *d = nullptr;
-  if (hipMalloc(&d, sizeof(int2) * std::max<size_t>(v.size(), 1)) != hipSuccess) { rsg_fail(errbuf, "hipMalloc tile list"); return nullptr; }
+  if (rsg_dev_malloc(&d, sizeof(int2) * std::max<size_t>(v.size(), 1)) != hipSuccess) { rsg_fail(errbuf, "hipMalloc tile list"); return nullptr; }
   if (!v.empty() && hipMemcpy(d, v.data(), sizeof(int2) * v.size(), hipMemcpyHostToDevice) != hipSuccess) { rsg_fail(errbuf, "tile list copy"); return nullptr; }
   cache[key] = std::make_pair(d, (int)v.size());
   *ntiles = (int)v.size();

@@ -103,7 +103,7 @@ struct DevMem {
   template <typename T> bool get(T **out, size_t count)
   {
     void *q = nullptr;
-    if (hipMalloc(&q, sizeof(T) * (count ? count : 1)) != hipSuccess) return false;
+    if (rsg_dev_malloc(&q, sizeof(T) * (count ? count : 1)) != hipSuccess) return false;
     p.push_back(q); *out = (T *)q; return true;
   }
 };

@@ -375,7 +375,7 @@ int ensure_part(rsg_mlp *m, int64_t nblk, char *errbuf)
   if (m->part_blocks >= nblk) return RSG_OK;
   if (m->d_part) hipFree(m->d_part);
   m->d_part = nullptr; m->part_blocks = 0;
-  HIPCHK(hipMalloc(&m->d_part, sizeof(float) * (size_t)(nblk * (m->P + 1))));
+  HIPCHK(rsg_dev_malloc(&m->d_part, sizeof(float) * (size_t)(nblk * (m->P + 1))));
   m->part_blocks = nblk;
   return RSG_OK;
 }
@@ -415,10 +415,10 @@ extern "C" int rsg_mlp_create(rsg_ctx *c, int nl, const int *dims, uint64_t seed
     }
   }
   const size_t pb = sizeof(float) * (size_t)m->P;
-  if (hipMalloc(&m->d_p, pb) != hipSuccess || hipMalloc(&m->d_m, pb) != hipSuccess ||
-      hipMalloc(&m->d_v, pb) != hipSuccess || hipMalloc(&m->d_g, pb) != hipSuccess ||
-      hipMalloc(&m->d_wb, sizeof(uint16_t) * (size_t)(m->P + 16)) != hipSuccess ||
-      hipMalloc(&m->d_scale, sizeof(float) * 2 * (size_t)(dims[0] + dims[nl])) != hipSuccess ||
+  if (rsg_dev_malloc(&m->d_p, pb) != hipSuccess || rsg_dev_malloc(&m->d_m, pb) != hipSuccess ||
+      rsg_dev_malloc(&m->d_v, pb) != hipSuccess || rsg_dev_malloc(&m->d_g, pb) != hipSuccess ||
+      rsg_dev_malloc(&m->d_wb, sizeof(uint16_t) * (size_t)(m->P + 16)) != hipSuccess ||
+      rsg_dev_malloc(&m->d_scale, sizeof(float) * 2 * (size_t)(dims[0] + dims[nl])) != hipSuccess ||
       hipMemcpy(m->d_p, h.data(), pb, hipMemcpyHostToDevice) != hipSuccess) {
     rsg_mlp_destroy(c, m);
     return rsg_fail(errbuf, "rsg_mlp_create: device allocation failed");
@@ -536,7 +536,7 @@ extern "C" int rsg_mlp_forward(rsg_ctx *c, rsg_mlp *m, const float *x, int64_t B
     if (m->d_io) hipFree(m->d_io);
     if (m->h_io) hipHostFree(m->h_io);
     m->d_io = m->h_io = nullptr; m->io_cap = 0;
-    HIPCHK(hipMalloc(&m->d_io, xb + yb));
+    HIPCHK(rsg_dev_malloc(&m->d_io, xb + yb));
     HIPCHK(hipHostMalloc((void **)&m->h_io, xb + yb, hipHostMallocDefault));
     m->io_cap = xb + yb;
   }
@@ -567,8 +567,8 @@ extern "C" int rsg_mlp_grad(rsg_ctx *c, rsg_mlp *m, const float *x, const float 
   if (ensure_part(m, nblk, errbuf) != RSG_OK) return RSG_FAIL;
   float *d_x = nullptr, *d_t = nullptr; double *d_l = nullptr;
   const size_t xb = sizeof(float) * (size_t)(B * m->dims[0]), tb = sizeof(float) * (size_t)(B * m->dims[m->nl]);
-  HIPCHK(hipMalloc(&d_x, xb));
-  if (hipMalloc(&d_t, tb) != hipSuccess || hipMalloc(&d_l, sizeof(double)) != hipSuccess) {
+  HIPCHK(rsg_dev_malloc(&d_x, xb));
+  if (rsg_dev_malloc(&d_t, tb) != hipSuccess || rsg_dev_malloc(&d_l, sizeof(double)) != hipSuccess) {
     hipFree(d_x); hipFree(d_t);
     return rsg_fail(errbuf, "rsg_mlp_grad: out of device memory");
   }
@@ -612,9 +612,9 @@ extern "C" int rsg_mlp_train(rsg_ctx *c, rsg_mlp *m, const float *x, const float
   if (ensure_part(m, nblk, errbuf) != RSG_OK) return RSG_FAIL;
   const size_t xb = sizeof(float) * (size_t)(n * m->dims[0]), tb = sizeof(float) * (size_t)(n * m->dims[m->nl]);
   float *d_x = nullptr, *d_t = nullptr; int *d_idx = nullptr; double *d_loss = nullptr;
-  if (hipMalloc(&d_x, xb) != hipSuccess || hipMalloc(&d_t, tb) != hipSuccess ||
-      hipMalloc(&d_idx, sizeof(int) * (size_t)n) != hipSuccess ||
-      hipMalloc(&d_loss, sizeof(double) * (size_t)steps) != hipSuccess) {
+  if (rsg_dev_malloc(&d_x, xb) != hipSuccess || rsg_dev_malloc(&d_t, tb) != hipSuccess ||
+      rsg_dev_malloc(&d_idx, sizeof(int) * (size_t)n) != hipSuccess ||
+      rsg_dev_malloc(&d_loss, sizeof(double) * (size_t)steps) != hipSuccess) {
     hipFree(d_x); hipFree(d_t); hipFree(d_idx); hipFree(d_loss);
     return rsg_fail(errbuf, "rsg_mlp_train: out of device memory");
   }

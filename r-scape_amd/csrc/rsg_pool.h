@@ -12,7 +12,8 @@
 // R-scape's own call: 236 us with them, 174 us without).  A block put back is handed out again for
 // a request of its size class; at most RSG_POOL_KEEP bytes are kept (the rest, and blocks over
 // RSG_POOL_BLOCK, go back to the device at once), all of them are given back with the context, and
-// by every pool when an allocation of the library fails.  Any thread may call.
+// by every pool when a device allocation of the library fails (rsg_dev_malloc makes them all).  Any
+// thread may call.
 // A pool does not wait for the device: its user keeps one of two rules.  `tmp` of a context holds
 // blocks that only work on that context's stream touches (RsgTmp), so stream order covers their
 // reuse; `pool` holds blocks of alignments, which any context may have used: they are put back
@@ -34,5 +35,7 @@ private:
   size_t kept = 0;
   bool open = true;
 };
-// hipMalloc; when it fails, again after every pool has given back its idle blocks
+// Every device allocation of the library: hipMalloc; when the device is full, again after every pool has
+// given back its idle blocks
 hipError_t rsg_dev_malloc(void **p, size_t bytes);
+template <typename T> static inline hipError_t rsg_dev_malloc(T **p, size_t bytes) { return rsg_dev_malloc((void **)p, bytes); }

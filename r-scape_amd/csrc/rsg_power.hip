@@ -98,7 +98,7 @@ struct Buf {
   template <typename T> bool get(T **o, size_t n)
   {
     void *q = nullptr;
-    if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) return false;
+    if (rsg_dev_malloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) return false;
     p.push_back(q); *o = (T *)q;
     return true;
   }
@@ -238,7 +238,7 @@ extern "C" int rsg_power_SPAIR_Create(rsg_ctx *c, rsg_msa *m, const int *msamap,
   std::vector<double4> sum((size_t)std::max<int64_t>(dim, 1));
   if (dim > 0) {
     double4 *d_sum = nullptr;
-    HIPCHK(hipMalloc(&d_sum, sizeof(double4) * (size_t)dim));
+    HIPCHK(rsg_dev_malloc(&d_sum, sizeof(double4) * (size_t)dim));
     const dim3 g((unsigned)((L * L + 255) / 256));
     if (m->cnt_kind == CNT_U16)      hipLaunchKernelGGL(k_pair_summary<CNT_U16>, g, dim3(256), 0, c->stream, m->d_cnt, L, rsg_count_wsum(m), d_sum);
     else if (m->cnt_kind == CNT_U32) hipLaunchKernelGGL(k_pair_summary<CNT_U32>, g, dim3(256), 0, c->stream, m->d_cnt, L, rsg_count_wsum(m), d_sum);

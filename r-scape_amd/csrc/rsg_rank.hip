@@ -214,7 +214,7 @@ static int ensure_rank(rsg_ctx *c, char *errbuf)
 {
   if (c->h_rank) return RSG_OK;
   if (!c->d_rank) {
-    HIPCHK(hipMalloc(&c->d_rank, RANK_SLICES + RANK_LISTB + RANK_COUNTS + RANK_DENSEB));
+    HIPCHK(rsg_dev_malloc(&c->d_rank, RANK_SLICES + RANK_LISTB + RANK_COUNTS + RANK_DENSEB));
     c->rank_dirty = RANK_DENSE;
   }
   HIPCHK(hipHostMalloc(&c->h_rank, sizeof(unsigned long long) * RANK_WIN + RANK_LISTB + 64, hipHostMallocDefault));
@@ -536,7 +536,7 @@ extern "C" int rsg_cov_Hits(rsg_ctx *c, rsg_msa *m, double thresh, int cap, int 
     if (c->d_hits) hipFree(c->d_hits);
     if (c->h_hits) hipHostFree(c->h_hits);
     c->d_hits = c->h_hits = nullptr; c->hits_cap = 0;
-    HIPCHK(hipMalloc(&c->d_hits, (sizeof(double2) + sizeof(int2)) * dcap));
+    HIPCHK(rsg_dev_malloc(&c->d_hits, (sizeof(double2) + sizeof(int2)) * dcap));
     HIPCHK(hipHostMalloc(&c->h_hits, (sizeof(double2) + sizeof(int2)) * dcap, hipHostMallocDefault));
     c->hits_cap = dcap;
   }

@@ -172,9 +172,9 @@ __global__ void k_cdf_list(const double *__restrict__ model, const double *__res
 extern "C" int rsg_gtr_cdf(rsg_ctx *c, const double *model, int64_t nt, const double *t, uint32_t *cdf, char *errbuf)
 {
   double *d_m = nullptr, *d_t = nullptr; uint32_t *d_c = nullptr;
-  HIPCHK(hipMalloc(&d_m, sizeof(double) * 40));
-  HIPCHK(hipMalloc(&d_t, sizeof(double) * (size_t)std::max<int64_t>(nt, 1)));
-  HIPCHK(hipMalloc(&d_c, sizeof(uint32_t) * 12 * (size_t)std::max<int64_t>(nt, 1)));
+  HIPCHK(rsg_dev_malloc(&d_m, sizeof(double) * 40));
+  HIPCHK(rsg_dev_malloc(&d_t, sizeof(double) * (size_t)std::max<int64_t>(nt, 1)));
+  HIPCHK(rsg_dev_malloc(&d_c, sizeof(uint32_t) * 12 * (size_t)std::max<int64_t>(nt, 1)));
   HIPCHK(hipMemcpy(d_m, model, sizeof(double) * 40, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(d_t, t, sizeof(double) * (size_t)nt, hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_cdf_list, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, c->stream, d_m, d_t, nt, d_c);
@@ -448,7 +448,7 @@ struct SimBuffers {
   template <typename T> bool get(T **out, size_t count)
   {
     void *q = nullptr;
-    if (hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return false;
+    if (rsg_dev_malloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return false;
     p.push_back(q); *out = (T *)q;
     return true;
   }
@@ -509,7 +509,7 @@ int rsg_sim_one(rsg_ctx *c, const rsg_null_job *job, const uint8_t *root, uint8_
   HIPCHK(hipSetDevice(c->device));
   if (job->nleaf < 2 || job->alen < 1) return rsg_fail(errbuf, "simulation needs >= 2 leaves and >= 1 column");
   uint8_t *d_leaves = nullptr;
-  HIPCHK(hipMalloc(&d_leaves, (size_t)(job->nleaf * job->alen)));
+  HIPCHK(rsg_dev_malloc(&d_leaves, (size_t)(job->nleaf * job->alen)));
   int64_t off = 0;
   int rc = rsg_simulate_device(c, 1, &job->nleaf, &job->alen, job->left, job->right, job->ld, job->rd,
                                job->model, &job->seed, &job->stream, &job->gapfrac, d_leaves, &off, errbuf, root);

@@ -1,5 +1,7 @@
 """Pools of device blocks: their rules on the CPU, against a device of counted bytes (tests/c/pool.cpp)."""
+import glob
 import os
+import re
 import subprocess
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -15,3 +17,16 @@ def test_pool_rules(tmp_path):
                            "-o", exe])
     r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.splitlines()[-1] == "threads ok", r.stdout + r.stderr
+
+
+def test_every_device_allocation_reclaims_idle_blocks():
+    """What the pools keep must not make another allocation of the library fail: device memory is
+    allocated through rsg_dev_malloc (pressure case above) and nowhere else."""
+    direct = []
+    for path in sorted(glob.glob(os.path.join(CSRC, "*"))):
+        if os.path.basename(path) == "rsg_pool.hip":
+            continue
+        for n, line in enumerate(open(path), 1):
+            if re.search(r"\bhip(Ext|Pitched)?Malloc(WithFlags|Managed|Pitch|Async)?\s*\(", line.split("//")[0]):
+                direct.append("%s:%d" % (os.path.basename(path), n))
+    assert not direct, direct
