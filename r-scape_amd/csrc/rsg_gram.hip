@@ -918,6 +918,8 @@ extern "C" const char *rsg_gram_shape_name(int s) { return (s >= 1 && s <= kNSha
 static const int2 *tile_list(int device, int64_t L, int BI, int BJ, int *ntiles, char *errbuf)
 {
   static std::map<std::tuple<int, int64_t, int, int>, std::pair<int2 *, int>> cache;
+  static std::mutex mu;                                 // contexts of several threads
+  std::lock_guard<std::mutex> lk(mu);
   auto key = std::make_tuple(device, L, BI, BJ);
   auto it = cache.find(key);
   if (it != cache.end()) { *ntiles = it->second.second; return it->second.first; }
@@ -929,7 +931,7 @@ static const int2 *tile_list(int device, int64_t L, int BI, int BJ, int *ntiles,
       if (bi * BI < jmax) v.push_back(make_int2((int)bi, (int)bj));
     }
   int2 *d = nullptr;
-  if (rsg_dev_malloc(&d, sizeof(int2) * std::max<size_t>(v.size(), 1)) != hipSuccess) { rsg_fail(errbuf, "hipMalloc tile list"); return nullptr; }
+  if (rsg_dev_malloc(&d, sizeof(int2) * std::max<size_t>(v.size(), 1)) != hipSuccess) { rsg_fail(errbuf, "tile list: out of device memory"); return nullptr; }
   if (!v.empty() && hipMemcpy(d, v.data(), sizeof(int2) * v.size(), hipMemcpyHostToDevice) != hipSuccess) { rsg_fail(errbuf, "tile list copy"); return nullptr; }
   cache[key] = std::make_pair(d, (int)v.size());
   *ntiles = (int)v.size();
