@@ -86,6 +86,11 @@ int         rsg_ctx_set_batch_persistent(rsg_ctx *ctx, int on);
  * host memory before they synchronise the stream, which they do in any case (default 0 microseconds: no
  * spin).  Results are the same either way (no reference counterpart). */
 int         rsg_ctx_set_stamp_wait(rsg_ctx *ctx, int microseconds);
+/* Gives the device memory the context keeps for later calls, and nobody uses now, back to the device
+ * (blocks of destroyed alignments and of finished calls, at most 2 GiB).  The library does so by
+ * itself when one of its own allocations does not fit; a program that shares the device with other
+ * allocators may call it any time (no reference counterpart). */
+int         rsg_ctx_trim(rsg_ctx *ctx);
 /* Counter calibration (no reference counterpart): runs the plain copy kernel
  * k_copy_probe over `bytes` (multiple of 16) three times, reading and writing `bytes` per
  * launch, so HBM counters of other kernels can be converted to bytes. */

@@ -59,6 +59,7 @@ def _declare(L):
         "rsg_ctx_set_gram_split": (i32, [vp, i32]),
         "rsg_ctx_set_batch_persistent": (i32, [vp, i32]),
         "rsg_ctx_set_stamp_wait": (i32, [vp, i32]),
+        "rsg_ctx_trim": (i32, [vp]),
         "rsg_ctx_graph_reuses": (i32, [vp]),
         "rsg_msa_create": (i32, [vp, vp, vp, i64, i64, C.POINTER(vp), cp]),
         "rsg_msa_update": (i32, [vp, vp, vp, vp, cp]),
@@ -257,6 +258,11 @@ class Context:
         """How long a scoring call spins on its completion stamp before it synchronises the
         stream (0, the default: not at all)."""
         self.L.rsg_ctx_set_stamp_wait(self.h, int(microseconds))
+
+    def trim(self):
+        """Give the device memory kept for later calls (blocks of closed alignments and finished
+        calls, at most 2 GiB) back to the device."""
+        self.L.rsg_ctx_trim(self.h)
 
     def graph_reuses(self):
         """Batched-null calls that replayed the context's cached graph without a new capture."""
