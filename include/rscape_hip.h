@@ -73,6 +73,9 @@ int         rsg_ctx_set_gram_shape(rsg_ctx *ctx, int shape);
  * reads gram_tiles.tsv next to itself on first use; this replaces that table for the process.
  * Sizes without an entry (and shape 0 contexts only) use the built-in choice. */
 int         rsg_gram_tiles_load(const char *path, char *errbuf);
+/* The shape a unit-weight Gram of this size takes: the context's, else the table's, else the built-in
+ * choice (ctx may be NULL: no shape set, 256 compute units). */
+int         rsg_gram_shape_for(const rsg_ctx *ctx, int64_t nseq, int64_t alen);
 /* 1 (default): when the tile count leaves a last partial wave of work groups, those tiles
  * are split along the sequence axis over the idle CUs and their partial counts summed
  * (integers, so the result is identical); 0: one work group per tile. */

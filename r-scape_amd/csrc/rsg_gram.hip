@@ -1097,21 +1097,26 @@ static int table_shape(int64_t N, int64_t L)
   return it == g_tiles.end() ? 0 : it->second;
 }
 
-static int pick_shape(const rsg_ctx *c, const rsg_msa *m)
+// The shape of a unit-weight Gram: the caller's, else the table's, else by rule.  (A line of the table
+// counts for its whole bucket: 32 x 32-column tiles, measured at 768 columns on launch_fp4_deep, also
+// past its 992 columns, where they cost at most a few per cent: 26.7 and 27.8 us, 71.3 and 68.1 against
+// 64 x 32 at 3072 and 12288 x 1008.)
+static int pick_shape(const rsg_ctx *c, int64_t N, int64_t L)
 {
-  int s = c->gram_shape;
+  int s = c ? c->gram_shape : 0;
   if (s >= 1 && s <= kNShapes) return s;
-  // 32 x 32-column tiles that fit the device at once go to launch_fp4_deep, whose range ends inside a
-  // bucket of the table
-  const int64_t nb = (m->L + 31) / 32;
-  const bool deep = nb * (nb + 1) / 2 <= 2 * (c->ncu > 0 ? c->ncu : 256);
-  s = table_shape(m->N, m->L);
-  if (s >= 1 && s <= kNShapes && !(s == 4 && !deep && m->N >= 1024)) return s;
+  s = table_shape(N, L);
+  if (s >= 1 && s <= kNShapes) return s;
   // sizes outside the table: 64 x 32-column tiles of four waves with 512-sequence K tiles win or tie
   // at N >= 1536 (two work groups per CU, so one's epilogue runs under the other's K loop); below
-  // ~1000 sequences (a few K tiles) 32 x 32 tiles of two waves are as fast; few tiles: as there
-  return (m->N < 1024 || (deep && m->N <= 16384)) ? 4 : 7;
+  // ~1000 sequences (a few K tiles) 32 x 32 tiles of two waves are as fast; where those fit the device at
+  // once launch_fp4_deep takes them
+  const int64_t nb = (L + 31) / 32;
+  const bool deep = nb * (nb + 1) / 2 <= 2 * (c && c->ncu > 0 ? c->ncu : 256);
+  return (N < 1024 || (deep && N <= 16384)) ? 4 : 7;
 }
+
+extern "C" int rsg_gram_shape_for(const rsg_ctx *c, int64_t N, int64_t L) { return pick_shape(c, N, L); }
 
 int rsg_gram_counts_fp4(rsg_ctx *c, rsg_msa *m, void *out, int kind, double *pm_part, int *pmflag, char *errbuf)
 {
@@ -1120,7 +1125,7 @@ int rsg_gram_counts_fp4(rsg_ctx *c, rsg_msa *m, void *out, int kind, double *pm_
     return (m->L >= 768) ? launch_fp4<2, 2, 512, CNT_U32>(c, m, out, nullptr, nullptr, errbuf)
                          : launch_fp4<1, 1, 256, CNT_U32>(c, m, out, nullptr, nullptr, errbuf);
   if (kind != CNT_U16) return rsg_fail(errbuf, "gram: bad record kind %d", kind);
-  switch (pick_shape(c, m)) {
+  switch (pick_shape(c, m->N, m->L)) {
   case 1: return launch_fp4<2, 2, 256, CNT_U16>(c, m, out, pm_part, pmflag, errbuf);
   case 2: return launch_fp4<2, 2, 128, CNT_U16>(c, m, out, pm_part, pmflag, errbuf);
   case 3: return launch_fp4<2, 2, 512, CNT_U16>(c, m, out, pm_part, pmflag, errbuf);

@@ -56,6 +56,7 @@ def _declare(L):
         "rsg_gram_shape_name": (cp, [i32]),
         "rsg_ctx_set_gram_shape": (i32, [vp, i32]),
         "rsg_gram_tiles_load": (i32, [cp, cp]),
+        "rsg_gram_shape_for": (i32, [vp, i64, i64]),
         "rsg_ctx_set_gram_split": (i32, [vp, i32]),
         "rsg_ctx_set_batch_persistent": (i32, [vp, i32]),
         "rsg_ctx_set_stamp_wait": (i32, [vp, i32]),

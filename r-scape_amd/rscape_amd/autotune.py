@@ -106,13 +106,14 @@ def main():
         return
     sizes = [(n, l) for n in GRID_N for l in GRID_L] if a.grid else [(a.N, a.L)]
     ctx = Context(0)
+    lib().rsg_gram_tiles_load(os.devnull.encode(), None)       # no table: the built-in choices
     tab, notes = read_table(a.out), {}
     for N, L in sizes:
         ax = synth.random_msa(N, L, np.random.default_rng(N + L), gap=0.1)
         res = sweep(ctx, ax, a.reps)
         ops = 2 * 16 * N * L * (L - 1) / 2
         best = min(res, key=lambda s: res[s][1])
-        dflt = res[7 if N >= 1024 else 4][1]
+        dflt = res[lib().rsg_gram_shape_for(ctx.h, N, L)][1]
         print("N=%d L=%d best %d %s %.4f ms (%.0f TOP/s); built-in choice %.4f ms" %
               (N, L, best, res[best][0], res[best][1], ops / (res[best][1] * 1e-3) / 1e12, dflt), flush=True)
         tab[bucket(N, L)] = best

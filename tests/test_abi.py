@@ -116,6 +116,28 @@ def test_gram_tiles_table_load(tmp_path):
         assert {autotune.bucket(n, l) for n in autotune.GRID_N for l in autotune.GRID_L} <= set(tab)
 
 
+def test_gram_tiles_table_is_followed(tmp_path):
+    """A line of the table decides the shape of every size of its bucket, whatever the built-in rule
+    would take (and it is the rule's choice that stands without a line); the committed table's too."""
+    from rscape_amd import autotune
+    L = R.lib()
+    err = C.create_string_buffer(256)
+    try:
+        assert L.rsg_gram_tiles_load(os.devnull.encode(), err) == 0
+        rule = {(n, l): L.rsg_gram_shape_for(None, n, l) for n in (1, 1023, 1024, 1500, 16384, 16385, 60000)
+                for l in (2, 992, 993, 1024, 1500, 5000)}
+        assert all(s == (4 if n < 1024 or (l <= 992 and n <= 16384) else 7) for (n, l), s in rule.items())
+        path = tmp_path / "t.tsv"
+        for shape in (4, 7, 3):
+            autotune.write_table({autotune.bucket(n, l): shape for n, l in rule}, str(path))
+            assert L.rsg_gram_tiles_load(str(path).encode(), err) == 0
+            assert {L.rsg_gram_shape_for(None, n, l) for n, l in rule} == {shape}
+    finally:
+        assert L.rsg_gram_tiles_load(autotune.TABLE.encode(), err) == 0, err.value
+    for (a, b), shape in autotune.read_table().items():
+        assert L.rsg_gram_shape_for(None, 2 ** a, 2 ** b) == L.rsg_gram_shape_for(None, 2 ** (a - 1) + 1, 2 ** (b - 1) + 1) == shape
+
+
 def test_autotune_table_from_sweep_lines(tmp_path):
     """The table rebuilt from printed sweep lines: one entry per bucket, later lines win, other
     lines ignored."""
