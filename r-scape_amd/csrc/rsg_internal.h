@@ -402,7 +402,7 @@ double *rsg_pm32_scratch(rsg_ctx *c, int64_t L, char *errbuf);
 int rsg_stat(rsg_ctx *c, rsg_msa *m, int base, int cls, const double *allow16, int prec, char *errbuf);
 int rsg_raf(rsg_ctx *c, rsg_msa *m, int rafs, const double *allow16, char *errbuf);
 int rsg_correct(rsg_ctx *c, rsg_msa *m, int actype, int shiftnonneg, char *errbuf);
-int rsg_reserve_scratch(rsg_ctx *c, int64_t L, char *errbuf);
+int rsg_reserve_scratch(rsg_ctx *c, int64_t L, bool pm_pass, char *errbuf);
 int rsg_minmax(rsg_ctx *c, rsg_msa *m, char *errbuf);
 int rsg_upload_weights_bf16(rsg_ctx *c, rsg_msa *m, int nsplit, char *errbuf);
 int64_t rsg_npad(int64_t N);

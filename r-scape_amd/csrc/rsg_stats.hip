@@ -19,11 +19,12 @@ static int ensure_red(rsg_ctx *c, size_t n, char *errbuf);
 #define RSG_MINMAX_BLOCKS 512   // partials of k_minmax_upper (RAF / RAFS extremes)
 
 // Reduction scratch large enough for every stage of one scoring of an L-column alignment
-// (sized before a deferred chain, so no stage reallocates it while earlier work is queued).
-int rsg_reserve_scratch(rsg_ctx *c, int64_t L, char *errbuf)
+// (sized before a deferred chain, so no stage reallocates it while earlier work is queued).  pm_pass: the
+// marginals take a pass of their own over the records (the Gram leaves no partials of them).
+int rsg_reserve_scratch(rsg_ctx *c, int64_t L, bool pm_pass, char *errbuf)
 {
   const int64_t nbt = (L + 63) / 64, nb = (L + 31) / 32;
-  const size_t need = std::max<size_t>({(size_t)(pm_npi(nbt) + pm_npj(nbt)), (size_t)(2 * pm32_n(nb)),
+  const size_t need = std::max<size_t>({pm_pass ? (size_t)(pm_npi(nbt) + pm_npj(nbt)) : 0, (size_t)(2 * pm32_n(nb)),
                                         (size_t)(4 * nb * (nb + 1) + 8 + 4 * L), (size_t)(2 * L + 8),
                                         (size_t)(2 * RSG_MINMAX_BLOCKS + 8)});
   return ensure_red(c, need, errbuf);

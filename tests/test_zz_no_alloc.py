@@ -93,6 +93,30 @@ def test_noalloc_matches_cov_calculate(ctx):
         d_cov.free()
 
 
+@pytest.mark.parametrize("N,L,covtype,prec", [(1, 2, "GTp", R.STAT_FP64), (30, 1, "GT", R.STAT_FP64),
+                                              (65, 768, "MIgp", R.STAT_FP32), (65, 769, "MIgp", R.STAT_FP32),
+                                              (130, 992, "GTp", R.STAT_FP64), (130, 993, "GTp", R.STAT_FP64),
+                                              (257, 1024, "CHIa", R.STAT_FP64), (4096, 1024, "GTp", R.STAT_FP64)])
+def test_noalloc_to_its_limits(ctx, N, L, covtype, prec):
+    """Up to RSG_NA_MAXN sequences and RSG_NA_MAXL columns, on either side of where the Gram's tiles
+    stop fitting the device at once (992 columns): rsg_cov_Calculate's scores bit for bit."""
+    ax = synth.random_msa(N, L, np.random.default_rng(N + L), gap=0.1)
+    m = ctx.msa(ax)
+    mn0, mx0 = m.calculate(covtype, prec=prec)
+    ref = m.get_cov()[0]
+    m.close()
+    d_ax, d_cov = DevBuf(N * L), DevBuf(8 * L * L)
+    try:
+        d_ax.put(ax)
+        rc, mn, mx, err = noalloc(ctx, d_ax, N, L, d_cov, covtype, prec)
+        assert rc == 0, err
+        assert np.array_equal(d_cov.get((L, L), np.float64), ref)
+        assert (mn, mx) == (mn0, mx0)
+    finally:
+        d_ax.free()
+        d_cov.free()
+
+
 @pytest.mark.parametrize("covtype", ["GT", "GTp", "GTa"])
 def test_noalloc_stamp_waits(ctx, covtype):
     """The chain's three ends (the statistic's own extremes, APC, ASC) with the completion stamp waited
