@@ -19,12 +19,13 @@
 //   1, 2 or 0; U's nibble (8 would be -0) is shifted right first, giving 2 or 0.  A product is
 //   one of 1/4 .. 4 exactly, the cell's unit; an accumulator starts at 2^23 units, where one
 //   FP32 ulp is one unit, so every sum is exact and the low mantissa bits are the count (up to
-//   65535 sequences; above, from 0, and the count is the accumulator over the unit).  The
-//   FP4 matrix rate is twice the int8 one (9.8 against 4.95 PFLOP/s measured from registers) and
-//   a panel holds half the bytes: the same Gram on int8 operands took 67 us at N = 5000 x L = 1500
-//   (44 us here, of which 18 at the full matrix rate; the rest is each tile's epilogue, the masks that
-//   share the issue slots with the matrix instructions, and the last, partial wave of tiles), 49 us
-//   at 4096 x 768 (20.7 us, k_gram_fp4_deep), 3.76 ms at 24576 x 6144 (2.1 ms, 7.0 PFLOP/s).
+//   65535 sequences; above, from 0, in K segments past FP4_EXACT sequences, and the count is the
+//   accumulator over the unit).  The FP4 matrix rate is twice the int8 one (9.8 against
+//   4.95 PFLOP/s measured from registers) and a panel holds half the bytes: the same Gram on int8
+//   operands took 67 us at N = 5000 x L = 1500 (44 us here, of which 18 at the full matrix rate;
+//   the rest is each tile's epilogue, the masks that share the issue slots with the matrix
+//   instructions, and the last, partial wave of tiles), 49 us at 4096 x 768 (20.7 us,
+//   k_gram_fp4_deep), 3.76 ms at 24576 x 6144 (2.1 ms, 7.0 PFLOP/s).
 // Weights: int8 limbs (v_mfma_i32_32x32x32_i8), or split-BF16 (w = hi + lo [+ lo2]) MFMA
 //   (v_mfma_f32_32x32x16_bf16); the i-side operand is 1.0 where the symbol matches, the j-side
 //   operand the split weight part; all parts accumulate into one FP32 accumulator.
@@ -206,6 +207,10 @@ __device__ __forceinline__ v4i and4(uint4 v, unsigned mk, int sh)
 {
   return (v4i){(int)((v.x >> sh) & mk), (int)((v.y >> sh) & mk), (int)((v.z >> sh) & mk), (int)((v.w >> sh) & mk)};
 }
+// Sequences an accumulator that starts at 0 takes (uint32 records): FP32 sums are exact to 2^24 units, a
+// unit per sequence at most.  More (the branches of a tree of millions of leaves) go in K segments of this
+// many, whose counts k_gram_fix adds as integers.
+#define FP4_EXACT (1 << 22)
 // FP4 value of symbol s's operand
 __host__ __device__ constexpr float fp4_unit(int s) { return s == 0 ? 0.5f : s == 1 ? 1.f : 2.f; }
 
@@ -993,7 +998,10 @@ static int launch_fp4(rsg_ctx *c, rsg_msa *m, void *out, double *pm_part, int *p
   }
   int ndp = ntiles, sbase = 1, sextra = 0;
   const int rem = ntiles % slots;
-  if (c->gram_split && ntiles < 4 * slots && rem > 0 && rem <= slots / 2 && nkt >= 2) {
+  if (OK == CNT_U32 && m->N > FP4_EXACT) {        // every tile in segments whose FP32 sums are exact
+    ndp = 0;
+    sbase = (int)(m->N / FP4_EXACT) + 1;
+  } else if (c->gram_split && ntiles < 4 * slots && rem > 0 && rem <= slots / 2 && nkt >= 2) {
     ndp = ntiles - rem;
     const int nsu = (int)std::min<int64_t>((int64_t)ncu, (int64_t)rem * nkt);
     sbase = nsu / rem; sextra = nsu % rem;

@@ -92,6 +92,22 @@ def test_fp4_counts_edges(ctx, shape, N):
     assert np.array_equal(got[iu], oracle.pair_counts(ax).reshape(L, L, 16)[iu].astype(float))
 
 
+@pytest.mark.parametrize("N", [2 ** 22, 2 ** 22 + 1, 2 ** 22 + 777])
+def test_fp4_counts_in_segments(ctx, N):
+    """Past 4194304 sequences the unit-weight Gram goes in K segments added as integers (one FP32 sum
+    is exact to 2^24): exact counts at either side, cells of N among them."""
+    L = 35
+    ax = np.tile(_msa(1021, L, 3), (N // 1021 + 1, 1))[:N]
+    for x in range(4):
+        ax[:, 8 * x] = ax[:, 8 * x + 3] = x
+    m = ctx.msa(ax)
+    m.probs(R.COUNTS_INT8)
+    got = m.counts().reshape(L, L, 16)
+    m.close()
+    iu = np.triu_indices(L, 1)
+    assert np.array_equal(got[iu], oracle.pair_counts(ax).reshape(L, L, 16)[iu].astype(float))
+
+
 @pytest.mark.parametrize("N", [1, 64, 65, 255, 321, 1030])
 @pytest.mark.parametrize("L", [2, 33, 703, 705, 992, 993])
 def test_gram_few_tiles(ctx, L, N):
