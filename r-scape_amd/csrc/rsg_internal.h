@@ -417,7 +417,7 @@ struct SimItem {
   int64_t col_blk0;       // first 64-column block of this item in the launch
   int64_t model_off;      // offset (doubles) of its 40-double GTR model
 };
-// Tree levels of a set of items: entries {item, internal node, first block within the level, 0}
+// Tree levels of a set of items: entries {item, internal node, left child, right child}
 // grouped by depth.
 // Host staging array without value-initialisation (every element is written before it is read).
 template <class T> struct HostArr {

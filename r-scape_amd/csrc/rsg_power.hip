@@ -7,7 +7,7 @@
 //     per column pair the branches that substitute at both columns (ndouble) or at either
 //     (njoin).  Here a branch x column code is formed on the device -- 0 a substitution, 1 no
 //     substitution, 4 neither (a gap or other code at an end, without --powergaps) -- and the
-//     pair counts are the int8 one-hot Gram of that branch alignment: ndouble = c[0][0],
+//     pair counts are the one-hot Gram of that branch alignment: ndouble = c[0][0],
 //     njoin = c[0][0] + c[0][1] + c[1][0] (counts of the 4 x 4 table of codes 0 and 1).
 //   power_Read (src/power.c:532-650), power_SPAIR_Create + power_SPAIR_AddMI (:65-217),
 //   cov_CreateHitList's selection (src/covariation.c:778-1006), cov_WriteHitList /
