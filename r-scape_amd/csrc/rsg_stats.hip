@@ -256,11 +256,16 @@ __global__ void __launch_bounds__(256) k_stat_strip(StatArgs A)
 
 // Whole or quarter tiles.  Quarters end sooner while the device is not full: GT in FP64 from uint16
 // records 6.3 against 8.6 us at 120 columns, 10.2 against 13.0 at 768, 33 against 39 at 2200, from
-// FP32 records 9.3 against 23.6, 23.8 against 35.8, 127 against 135 us.  Past 4096 tiles (2880
+// FP32 records 9.3 against 23.6, 23.8 against 35.8, 127 against 135 us; the other statistics and class C2
+// alike (at 2200 columns MIr 36 against 40, CHI 43 and 46, OMES 28 and 31, GT of C2 50 and 52, weighted
+// MIr 132 and 135, CHI 41 and 46; at 2880 all within 2% of whole tiles or ahead).  Past 4096 tiles (2880
 // columns) whole tiles' longer stores to the lower triangle win from uint16 records (104 against
-// 116 us at 3600, 215 against 239 at 5000; from FP32 records the two are equal), and half tiles in
-// FP32 (194 against 212 us at 5000 from FP32 records; quarters 20.4 against 21.7 at 1500).
+// 116 us at 3600, 215 against 239 at 5000; from FP32 records the two are equal).
+// In FP32 half tiles win sooner, from weighted records: quarters are ahead or even at 2400 columns (MIr 52
+// against 53, CHI 39 and 43, GT and MI 46 and 46), behind at 2500 (GT and MI 57.6 and 54) and 2880
+// (75 and 69); from uint16 records the two are within 2% throughout.
 #define STAT_STRIP_TILES 4096       // 90 tiles of 32 columns: 4095
+#define STAT_PART_TILES  2850       // FP32: 75 tiles of 32 columns
 template <typename T, int KIND, bool TAB, int TYPE, int CLS>
 static int launch_tiles(rsg_ctx *c, const StatArgs &A, int nb)
 {
@@ -315,7 +320,7 @@ static int launch_stat_f32_fixed(rsg_ctx *c, const StatArgs &A, int kind, int cl
   if (cls != RSG_C16 || (kind != CNT_U16 && kind != CNT_F32)) return 0;
   const int ntri = nb * (nb + 1) / 2;
   if constexpr (TYPE == RSG_GT || TYPE == RSG_MI || TYPE == RSG_MIg || TYPE == RSG_MIr || TYPE == RSG_CHI || TYPE == RSG_OMES) {
-    if (ntri <= STAT_STRIP_TILES) {
+    if (ntri <= STAT_PART_TILES) {
       const dim3 grid((unsigned)(4 * ntri));
       if (kind == CNT_U16) hipLaunchKernelGGL((k_stat_part<CNT_U16, TYPE, 1>), grid, dim3(256), 0, c->stream, A);
       else                 hipLaunchKernelGGL((k_stat_part<CNT_F32, TYPE, 1>), grid, dim3(256), 0, c->stream, A);

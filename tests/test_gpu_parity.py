@@ -302,6 +302,25 @@ def test_statistic_tile_parts(ctx, L):
         m.close()
 
 
+@pytest.mark.parametrize("L", [2400, 2401])
+def test_statistic_fp32_parts(ctx, L):
+    """FP32 statistics over quarter tiles (up to 2400 columns) and over half ones, within the
+    FP32 bound of the tests at other sizes of the FP64 statistic, and the matrix's own extremes."""
+    N = 24
+    ax = _msa(N, L, 78)
+    for wgt, mode in ((None, R.COUNTS_INT8), (np.random.default_rng(5).uniform(0.2, 2.0, N), R.COUNTS_W8)):
+        m = ctx.msa(ax, wgt)
+        m.probs(mode)
+        m.cov("GT", R.C16, prec=R.STAT_FP64)
+        ref = _upper(m.get_cov()[0], L)
+        m.cov("GT", R.C16, prec=R.STAT_FP32)
+        got, mn, mx = m.get_cov()
+        up = _upper(got, L)
+        assert _relerr(up, ref) < 1e-5
+        assert [mn, mx] == [up.min(), up.max()] and np.array_equal(got, got.T)
+        m.close()
+
+
 def test_gt_cwc_and_cselect(ctx):
     ax = _msa(6, 40, 3)            # nseq <= 8 -> CSELECT resolves to C2
     m = ctx.msa(ax)
