@@ -130,7 +130,8 @@ __global__ void __launch_bounds__(NT) k_fitch_up(const int4 *__restrict__ ent, i
 // 64 columns of all depths, 16 threads a node -- as many nodes as its threads hold at once: a wider
 // depth would go round on a few CUs -- and the depths follow each other behind its own barriers.
 // Bound by latency (a child's bytes, then the barrier): 1.4 us a depth, 25 us for 18 depths of 400
-// sequences of 203 columns, which took 66 with a launch each.
+// sequences of 203 columns, which took 66 with a launch each.  (Runs of 32 depths at most: of 8 a null of 20
+// replicates on a chain of 400 takes 2495 us in place of 2438, of 64 it takes 2426 with more kernel arguments.)
 #define FITCH_RUN_W 64
 #define FITCH_RUN_D 32
 struct UpRun { int n, lev[FITCH_RUN_D + 1]; };
@@ -656,8 +657,11 @@ static void fitch_down(rsg_ctx *c, const FitchPlan &P, const FitchDev &D, int R,
 }
 
 // Threads of a work group of the passes: enough for a dword (four columns) each, so that a row takes one
-// round of a pass's barriers.  1500 columns: 256 threads take a second round for 119 dwords (upward
-// pass 4.3 us a depth), 384 take one (3.5).  Past 2048 columns 256 threads go round.
+// round of a pass's barriers, 512 at most.  1500 columns: 256 threads take a second round for 119 dwords
+// (upward pass 4.3 us a depth), 384 take one (3.5).  Past 2048 columns the rounds go on at 512: a null of
+// 1000 sequences of 2049, 4096 and 9000 columns takes 366, 618 and 1956 us, with 256 threads 422, 727 and
+// 2208, with 384 389, 682 and 2067; ten of them at once, where a depth has work groups enough, 1227 and
+// 3231 us at 2049 and 4096 columns, with 256 threads 1225 and 3395.
 template <class F>
 static int fitch_width(int64_t L, F f)
 {
@@ -665,8 +669,7 @@ static int fitch_width(int64_t L, F f)
   if (L <= 512)  return f(std::integral_constant<int, 128>());
   if (L <= 1024) return f(std::integral_constant<int, 256>());
   if (L <= 1536) return f(std::integral_constant<int, 384>());
-  if (L <= 2048) return f(std::integral_constant<int, 512>());
-  return f(std::integral_constant<int, 256>());
+  return f(std::integral_constant<int, 512>());
 }
 
 template <int NT>
