@@ -340,12 +340,12 @@ __global__ void k_width_b(int ng, const int *__restrict__ gfirst, const int64_t 
 // Bins of every group in one pool: offsets by an exclusive scan over the groups (one block,
 // fixed order); a group that does not fit in the pool's cap bins is marked failed (its fit is
 // NaN, as for a group without a histogram).  Up to 1024 groups, one per thread, the geometry is
-// formed here, and of a few groups the bins are cleared here: two launches of 5 us less.
-#define HIST_LAYOUT_CLEAR 8
+// formed here: a launch of 5 us less.  (The bins of a few groups cleared here as well took the time
+// their launch takes, those of 32 and 200 groups 13 and 80 us more.)
 __global__ void __launch_bounds__(1024) k_hist_layout(int ng, HGeo *__restrict__ geo, int64_t cap,
                                                       const int *__restrict__ gfirst, const int64_t *__restrict__ desc,
                                                       const double *__restrict__ mm, double bmin, double w0, int hpts,
-                                                      double tol, unsigned long long *__restrict__ hist)
+                                                      double tol)
 {
   __shared__ int64_t sh[1024];
   const int T = 1024, tid = threadIdx.x;
@@ -367,12 +367,6 @@ __global__ void __launch_bounds__(1024) k_hist_layout(int ng, HGeo *__restrict__
     geo[g].off = off;
     off += geo[g].nb;
     if (off > cap) geo[g].ok = 0;
-  }
-  if (ng > HIST_LAYOUT_CLEAR) return;
-  __syncthreads();
-  for (int g = 0; g < ng; g++) {
-    if (!geo[g].ok) continue;
-    for (int b = tid; b < geo[g].nb; b += T) hist[geo[g].off + b] = 0ull;
   }
 }
 
@@ -751,9 +745,8 @@ static int null_batch_impl(rsg_ctx *c, const rsg_null_job *jobs, int nj, int cov
       hipLaunchKernelGGL(k_width_b, dim3((unsigned)((ng + 63) / 64)), dim3(64), 0, c->stream, ng, d_gfirst, d_desc, d_mm,
                          bmin, 0.05, 400, 1e-6, d_geo);
     hipLaunchKernelGGL(k_hist_layout, dim3(1), dim3(1024), 0, c->stream, ng, d_geo, pool, d_gfirst, d_desc, d_mm, bmin, 0.05, 400,
-                       1e-6, d_hist);
-    if (ng > HIST_LAYOUT_CLEAR)
-      hipLaunchKernelGGL(k_clear_bins, dim3((unsigned)std::min(ng, 4096)), dim3(256), 0, c->stream, ng, d_geo, d_hist);
+                       1e-6);
+    hipLaunchKernelGGL(k_clear_bins, dim3((unsigned)std::min(ng, 4096)), dim3(256), 0, c->stream, ng, d_geo, d_hist);
     hipLaunchKernelGGL(k_hist_b, dim3((unsigned)b_hist), dim3(1024), 0, c->stream, d_desc, M.m + M.off[M_HIST], d_cov, d_rows, actype, d_geo,
                        bmin, htarget, d_hist);
     hipLaunchKernelGGL(k_fit_b, dim3((unsigned)ng), dim3(1024), 0, c->stream, d_geo, d_hist, bmin, pmass, fracfit, doexpfit, d_fits);
