@@ -530,8 +530,9 @@ __device__ void pm_tile(const void *__restrict__ cnt, int64_t L, int nbt, int bi
 // blk = pm_tri(bi, bj, nb32).
 __host__ __device__ __forceinline__ int64_t pm32_n(int64_t nb32) { return pm_tri(nb32, nb32, nb32) * 32 * 4; }
 
-// 1 / (ns + 16e-10), correctly rounded as the division is: the division's own steps (two Newton steps,
-// a remainder step) without its scaling and special cases, which no ns in 1 .. 65535 needs
+// 1 / (ns + 16e-10) by Newton's iteration on the reciprocal and a final step from the remainder by FMA (P. W.
+// Markstein, Computation of elementary functions on the IBM RISC System/6000 processor, IBM J. Res.
+// Dev. 34, 1990): correctly rounded, checked against the division for every ns in 1 .. 65535.
 __device__ __forceinline__ double pm_inv(bool valid, int ns)
 {
 #pragma clang fp contract(off)
