@@ -174,6 +174,36 @@ def test_noalloc_leaves_no_work_behind():
         d_cov.free()
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_noalloc_beside_a_capture(ctx, mode):
+    """The call on its own stream while the caller captures another one (global, thread-local and
+    relaxed capture): it scores, and the capture ends with its graph."""
+    N, L = 200, 120
+    ax = synth.config(0, seed=6, N=N, L=L)["ax"]
+    m = ctx.msa(ax)
+    m.calculate("GTp")
+    ref = m.get_cov()[0]
+    m.close()
+    d_ax, d_cov = DevBuf(N * L), DevBuf(8 * L * L)
+    st, graph = C.c_void_p(), C.c_void_p()
+    h = hip()
+    try:
+        d_ax.put(ax)
+        assert h.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+        assert h.hipStreamBeginCapture(st, mode) == 0
+        rc, _, _, err = noalloc(ctx, d_ax, N, L, d_cov, "GTp", R.STAT_FP64)
+        assert h.hipStreamEndCapture(st, C.byref(graph)) == 0 and graph.value
+        assert rc == 0, err
+        assert np.array_equal(d_cov.get((L, L), np.float64), ref)
+    finally:
+        if graph.value:
+            h.hipGraphDestroy(graph)
+        if st.value:
+            h.hipStreamDestroy(st)
+        d_ax.free()
+        d_cov.free()
+
+
 def test_noalloc_rejects_oversize_and_unsupported(ctx):
     d = DevBuf(64)
     try:
