@@ -986,7 +986,8 @@ static int launch_fp4(rsg_ctx *c, rsg_msa *m, void *out, double *pm_part, int *p
   // K into one segment per CU, which run after the full tiles in the slots the first of them
   // free (the two work groups that share a CU finish far apart), then reduced (with many waves
   // the tail is small and the partial traffic costs more).  A CU holds 8 waves of this kernel
-  // (two per SIMD): 4 / (WI WJ) work groups.
+  // (two per SIMD): 4 / (WI WJ) work groups.  Of more tiles than CUs (half a wave of the smallest ones)
+  // some would be left without a segment.
   const int ncu = c->ncu > 0 ? c->ncu : 256;
   const int slots = std::max(ncu * 4 / (WI * WJ), 1);
   // whole K-tiles; when the sequences past the last whole one fit one 64-sequence k-step, that
@@ -1001,7 +1002,7 @@ static int launch_fp4(rsg_ctx *c, rsg_msa *m, void *out, double *pm_part, int *p
   if (OK == CNT_U32 && m->N > FP4_EXACT) {        // every tile in segments whose FP32 sums are exact
     ndp = 0;
     sbase = (int)(m->N / FP4_EXACT) + 1;
-  } else if (c->gram_split && ntiles < 4 * slots && rem > 0 && rem <= slots / 2 && nkt >= 2) {
+  } else if (c->gram_split && ntiles < 4 * slots && rem > 0 && rem <= std::min(slots / 2, ncu) && nkt >= 2) {
     ndp = ntiles - rem;
     const int nsu = (int)std::min<int64_t>((int64_t)ncu, (int64_t)rem * nkt);
     sbase = nsu / rem; sextra = nsu % rem;

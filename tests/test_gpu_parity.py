@@ -108,6 +108,37 @@ def test_fp4_counts_in_segments(ctx, N):
     assert np.array_equal(got[iu], oracle.pair_counts(ax).reshape(L, L, 16)[iu].astype(float))
 
 
+@pytest.mark.parametrize("shape,N,L", [(0, 600, 1601), (0, 600, 1728), (4, 513, 1632), (4, 513, 2180), (9, 1025, 1632), (9, 520, 720),
+                                       (1, 300, 1632), (7, 1100, 1632), (0, 65600, 720), (0, 65600, 767), (0, 40, 730)])
+def test_gram_every_tile_counted(ctx, shape, N, L):
+    """Every 32 x 32 block of pairs, where the last wave of tiles holds more of them than there are
+    compute units (the split along K deals a segment per unit: a tile may not go without one), with
+    uint16 records of the smallest tiles and uint32 ones, and tiles of other sizes: one pair per block
+    against its counts from the codes."""
+    ax = _msa(N, L, N + L)
+    ctx.set_gram_shape(shape)
+    try:
+        m = ctx.msa(ax)
+        m.probs(R.COUNTS_INT8)
+        got = m.counts().reshape(L, L, 16)
+        m.close()
+    finally:
+        ctx.set_gram_shape(0)
+    rng = np.random.default_rng(L)
+    bad = []
+    for bi in range(0, L, 32):
+        for bj in range(bi, L, 32):
+            j = int(rng.integers(max(bj, bi + 1), min(bj + 32, L))) if max(bj, bi + 1) < min(bj + 32, L) else -1
+            if j < 0:
+                continue
+            i = int(rng.integers(bi, min(bi + 32, j)))
+            ok = (ax[:, i] < 4) & (ax[:, j] < 4)
+            ref = np.bincount(4 * ax[ok, i].astype(int) + ax[ok, j], minlength=16)
+            if not np.array_equal(got[i, j], ref):
+                bad.append((bi // 32, bj // 32))
+    assert not bad, (len(bad), bad[:5])
+
+
 @pytest.mark.parametrize("N", [1, 64, 65, 255, 321, 1030])
 @pytest.mark.parametrize("L", [2, 33, 703, 705, 992, 993])
 def test_gram_few_tiles(ctx, L, N):
